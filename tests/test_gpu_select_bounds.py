@@ -135,3 +135,38 @@ def test_probability_topk_with_ties(dtype):
     top, scores = ops.select_topk_probs(probs.to(dev()), vis.to(dev()), k_sel, n_kv, return_scores=True)
     exp = ref.topk_positions(scores.cpu().numpy(), vis.numpy(), k_sel)
     np.testing.assert_array_equal(top.cpu().numpy(), exp)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("side", ["above", "below"])
+def test_scores_beyond_the_first_parts(side, dtype):
+    """Rows of 1024 in one channel, so that the first part of the split sees nothing of
+    8 in the others and 16 in place of 9. Above: five keys score 1550 (log2), all of it
+    beyond the first parts. Below: five keys score 4, of which the first parts see 1400."""
+    announce(f"bounded selection: scores beyond the first parts, {side} {dtype}")
+    gen = torch.Generator().manual_seed(21)
+    P, T = 3000, 64
+    q = torch.randn(1, 28, T, 128, generator=gen)
+    k = torch.randn(1, 4, P, 128, generator=gen)
+    if side == "above":
+        q[:, :, ::2] = 8
+        k[:, :, 100:600:100] = 12
+    else:
+        q[:, :, ::2, :100], q[:, :, ::2, 100:] = 9, 32
+        k[..., 127] *= 0.05
+        k[:, :, 100:600:100, :100], k[:, :, 100:600:100, 100:] = 16, -16.625
+    q[:, :, ::2, 127] = 1024
+    k[:, :, 100:600:100, 127] = 0
+    _check(q.to(dtype), k.to(dtype), P - T, torch.arange(P - T, dtype=torch.int32), 300)
+
+
+def test_scores_past_the_references_integers():
+    """Powers of two, which the first part holds whole, with scores of 1e11: the
+    reference, a float, steps by more than the exponents' range."""
+    announce("bounded selection: scores of 1e11")
+    gen = torch.Generator().manual_seed(22)
+    P, T = 3000, 64
+    q = torch.exp2(torch.randint(16, 19, (1, 28, T, 128), generator=gen).float())
+    k = torch.exp2(torch.randint(16, 19, (1, 4, P, 128), generator=gen).float())
+    k *= torch.randint(0, 2, k.shape, generator=gen) * 2 - 1
+    _check(q.to(torch.bfloat16), k.to(torch.bfloat16), P - T, torch.arange(P - T, dtype=torch.int32), 300)
