@@ -170,3 +170,15 @@ def test_scores_past_the_references_integers():
     k = torch.exp2(torch.randint(16, 19, (1, 4, P, 128), generator=gen).float())
     k *= torch.randint(0, 2, k.shape, generator=gen) * 2 - 1
     _check(q.to(torch.bfloat16), k.to(torch.bfloat16), P - T, torch.arange(P - T, dtype=torch.int32), 300)
+
+
+def test_fp16_elements_near_the_largest():
+    """fp16 elements from 65280 on, whose first part would round to 65536."""
+    announce("bounded selection: fp16 elements near the largest")
+    gen = torch.Generator().manual_seed(23)
+    P, T = 3000, 64
+    q = torch.randn(1, 28, T, 128, generator=gen)
+    q[..., 0] *= 1e-3
+    k = torch.randn(1, 4, P, 128, generator=gen)
+    k[:, :, 50:2500:50, 0] = torch.tensor([65280.0, 65472.0, 65504.0, -65504.0, 65248.0, -65280.0, 65312.0]).repeat(7)
+    _check(q.half(), k.half(), P - T, torch.arange(P - T, dtype=torch.int32), 300)
