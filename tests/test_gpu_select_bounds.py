@@ -182,3 +182,52 @@ def test_fp16_elements_near_the_largest():
     k = torch.randn(1, 4, P, 128, generator=gen)
     k[:, :, 50:2500:50, 0] = torch.tensor([65280.0, 65472.0, 65504.0, -65504.0, 65248.0, -65280.0, 65312.0]).repeat(7)
     _check(q.half(), k.half(), P - T, torch.arange(P - T, dtype=torch.int32), 300)
+
+
+@pytest.mark.parametrize("side", [1, -1])
+@pytest.mark.parametrize("shift", [1e-10, 3e-11])
+def test_tied_keys_next_to_a_close_one(side, shift):
+    """Two equal keys straddle the k-th place below a third that scores 1e-5 more, and
+    another key scores 1 + side x shift of theirs, closer than the split statistics'
+    error: rows of one kind weigh the tied keys, rows of the other kind that one, on
+    disjoint channels, so the two kinds' errors do not cancel."""
+    announce(f"bounded selection: tied keys next to a close one {side} {shift}")
+    gen = torch.Generator().manual_seed(24)
+    n_kv, T, P, D = 4, 64, 9000, 128
+    q = torch.zeros(1, n_kv, T, D)
+    q[:, :, ::2, :60] = torch.randn(1, n_kv, T // 2, 60, generator=gen) * 4 + 20
+    q[:, :, ::2, 60] = 2.0 ** -6
+    q[:, :, 1::2, 64:123] = torch.randn(1, n_kv, T // 2, 59, generator=gen) + 1
+    for c in range(5):                                     # fine channels of the second kind of row
+        q[:, :, 1::2, 123 + c] = 2.0 ** (-4 - 8 * c)
+    q = q.bfloat16()
+    k = torch.randn(1, n_kv, P, D, generator=gen)
+    k[..., :61] *= 0.03
+    k[:, :, 20:60:10] = 0
+    k[:, :, 20:50:10, :60] = 0.11
+    k[:, :, 20, 60] = 0.02
+    k = k.bfloat16()
+
+    def gap(g):                                            # of keys 30 and 50, in 64 bits
+        s = q[0, g].double() @ k[0, g].double().T / D ** 0.5
+        s.masked_fill_(torch.arange(P)[None] > P - T + torch.arange(T)[:, None], float("-inf"))
+        p = torch.softmax(s, -1).sum(0)
+        return (p[50] / p[30] - 1 - side * shift).item()
+
+    for g in range(n_kv):
+        # the close key: along the second kind's mean, then channel by channel nearer
+        for c, reach in [(slice(64, 123), 4.0)] + [(c, 64.0) for c in range(123, 128)]:
+            lo, hi, best = -reach, reach, (9.0, 0.0)
+            for _ in range(16):
+                mid = (lo + hi) / 2
+                k[0, g, 50, c] = mid
+                x = gap(g)
+                best = min(best, (abs(x), mid))
+                lo, hi = (mid, hi) if x < 0 else (lo, mid)
+            k[0, g, 50, c] = best[1]
+        assert abs(gap(g)) < shift / 4
+    vis = torch.arange(P - T, dtype=torch.int32)
+    scores = ops.select_topk(q.to(dev()), k.to(dev()), P - T, vis.to(dev()), 4, return_scores=True)[1].cpu()
+    above = {int((scores[g, :P - T] > scores[g, 20]).sum()) for g in range(n_kv)}
+    for k_sel in sorted({a + i for a in above for i in (1, 2, 3)}):
+        _check(q, k, P - T, vis, k_sel)
