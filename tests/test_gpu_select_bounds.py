@@ -231,3 +231,19 @@ def test_tied_keys_next_to_a_close_one(side, shift):
     above = {int((scores[g, :P - T] > scores[g, 20]).sum()) for g in range(n_kv)}
     for k_sel in sorted({a + i for a in above for i in (1, 2, 3)}):
         _check(q, k, P - T, vis, k_sel)
+
+
+@pytest.mark.parametrize("P", [2000, 16000])               # fp64 statistics; split ones, which leave it undecided
+def test_scores_equal_but_for_rounding(P):
+    """Pairs of keys whose scores are the same sums of the same terms in another order:
+    they differ in their last bits, by the order of the additions alone."""
+    announce(f"bounded selection: scores equal but for rounding, {P} keys")
+    gen = torch.Generator().manual_seed(25)
+    T, n = 40, (P - 40) // 2
+    q = torch.randn(1, 8, T, 128, generator=gen)
+    q[:, 1::2] = q[:, ::2].flip(-1)
+    k = torch.randn(1, 2, P, 128, generator=gen)
+    k[:, :, n:2 * n] = k[:, :, :n].flip(-1)
+    k[:, :, 2 * n:, 64:] = k[:, :, 2 * n:, :64].flip(-1)
+    for k_sel in range(101, 500, 26):
+        _check(q.bfloat16(), k.bfloat16(), P - T, torch.arange(2 * n, dtype=torch.int32), k_sel)
