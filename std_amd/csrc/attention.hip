@@ -1563,19 +1563,19 @@ attn_f32_kernel(const float* __restrict__ q, float* __restrict__ kc, float* __re
     const bool need_mask = key0 + 16 > kv_len || key0 + 15 > causal_off;
 #pragma unroll
     for (int rt = 0; rt < NT; ++rt) {
+      // the mask and the maximum are of the scaled scores: a scale may be 0 or negative
+      f32x4 x = s[rt] * scale_log2;
+      const int seen = min(kv_len - 1, lim[rt]) - (key0 + 4 * lg);   // last of the lane's keys that counts
       if (need_mask) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int key = key0 + 4 * lg + i;
-          s[rt][i] = key < kv_len && key <= lim[rt] ? s[rt][i] : -INFINITY;
-        }
+        for (int i = 0; i < 4; ++i) x[i] = i <= seen ? x[i] : -INFINITY;
       }
       // The running max follows every tile (one wave-uniform branch where a row's
       // rises), without the 16-bit kernels' slack, and the exponent is one fma: its
       // rounding is then that of a small difference where the large terms are. With
       // the slack and a rounded product the outputs were 5 to 35 % further from 64
       // bits (130 to 4106 keys).
-      const float lm = fmaxf(fmaxf(s[rt][0], s[rt][1]), fmaxf(s[rt][2], s[rt][3])) * scale_log2;
+      const float lm = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
       if (__ballot(lm > m_run[rt])) {
         const float m_new = fmaxf(m_run[rt], xor32_max(xor16_max(lm)));
         const float alpha = fast_exp2(m_run[rt] - m_new);
@@ -1586,6 +1586,10 @@ attn_f32_kernel(const float* __restrict__ q, float* __restrict__ kc, float* __re
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) s[rt][i] = fast_exp2(fmaf(s[rt][i], scale_log2, -m_run[rt]));
+      if (need_mask) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[rt][i] = i <= seen ? s[rt][i] : 0.f;
+      }
       l_run[rt] += (s[rt][0] + s[rt][1]) + (s[rt][2] + s[rt][3]);
     }
 #pragma unroll

@@ -1,11 +1,12 @@
 """The attention wrappers' short form check: what it does not take goes through
-every check and gives the same result or the same error."""
+every check and gives the same result or the same error; and any scale."""
 import numpy as np
 import pytest
 import torch
 
+from oracle import attention as ref
 from std_amd import ops
-from tests.gpu_helpers import announce, dev
+from tests.gpu_helpers import announce, assert_close, cache_buffer, dev
 
 pytestmark = pytest.mark.gpu
 
@@ -63,3 +64,22 @@ def test_streams_have_their_own_workspace():
     torch.cuda.current_stream().wait_stream(side)
     assert torch.equal(got, exp)
     assert ops._stream(q.device) == torch.cuda.current_stream().cuda_stream
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("scale", [0.0, -0.125])
+@pytest.mark.parametrize("q_len,kv_len", [(1, 70), (1, 300), (5, 70), (10, 333)])
+def test_any_scale(q_len, kv_len, scale, dtype):
+    """Scale 0 (the mean of the values seen) and a negative one, off the tile: the mask
+    and the running maximum are those of the scaled scores."""
+    announce(f"attention scale {scale} q={q_len} kv={kv_len} {dtype}")
+    gen = torch.Generator().manual_seed(q_len + kv_len)
+    q = torch.randn(1, 14, q_len, 128, generator=gen).to(dtype)
+    k, v = (torch.randn(1, 2, kv_len, 128, generator=gen).to(dtype) for _ in "kv")
+    exp = ref.verify_attention(q, k, v, scale=scale)
+    kb, vb = cache_buffer(k, kv_len + 30), cache_buffer(v, kv_len + 30)
+    assert_close(ops.verify_attention(q.to(dev()), kb[:, :, :kv_len], vb[:, :, :kv_len], scale=scale), exp, dtype)
+    new = [x[:, :, kv_len - q_len:].to(dev()) for x in (k, v)]
+    assert_close(ops.verify_attention_append(q.to(dev()), kb, vb, *new, kv_len, scale=scale), exp, dtype)
+    if q_len == 1:
+        assert_close(ops.gqa_decode(q.to(dev()), kb[:, :, :kv_len], vb[:, :, :kv_len], scale=scale), exp, dtype)
