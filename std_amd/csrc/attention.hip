@@ -1514,7 +1514,7 @@ attn_f32_kernel(const float* __restrict__ q, float* __restrict__ kc, float* __re
     for (int t = 0; t < 8; ++t) acc[rt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
-  // A tile's operands: keys past the cache's last re-read it (masked below).
+  // A tile's operands: keys past the cache's last re-read it (masked, and cleared in V, below).
   f32x4 kf[8], vf[4][2];
   auto load_k = [&](int t) {
     const int key = min(tile_key0(split, t, n_split) + 16 * w + ln, kv_len - 1);
@@ -1591,6 +1591,12 @@ attn_f32_kernel(const float* __restrict__ q, float* __restrict__ kc, float* __re
         for (int i = 0; i < 4; ++i) s[rt][i] = i <= seen ? s[rt][i] : 0.f;
       }
       l_run[rt] += (s[rt][0] + s[rt][1]) + (s[rt][2] + s[rt][3]);
+    }
+    if (key0 + 16 > kv_len) {                                     // no values: 0 times the last one's infinity is NaN
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) vf[j][c] = key0 + 4 * lg + j < kv_len ? vf[j][c] : f32x4{0.f, 0.f, 0.f, 0.f};
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j)

@@ -39,3 +39,19 @@ def test_f32_rows(n_q, n_kv, q_len, kv_len):
     assert torch.equal(out, again)
     assert torch.equal(kb[:, :, first:kv_len], nk) and torch.equal(vb[:, :, first:kv_len], nv)
     assert torch.isnan(kb[:, :, kv_len:]).all()
+
+
+@pytest.mark.parametrize("kv_len", [3, 70, 700])
+def test_f32_infinite_last_value(kv_len):
+    """The last key's value infinite in two columns, off the tile: infinite there for the
+    row that sees it, untouched elsewhere (rows past the cache's last are not values)."""
+    announce(f"fp32 infinite last value kv={kv_len}")
+    gen = torch.Generator().manual_seed(kv_len)
+    q = torch.randn(1, 7, 1, 128, generator=gen)
+    k, v = (torch.randn(1, 1, kv_len, 128, generator=gen) for _ in "kv")
+    exp = torch.from_numpy(ref.verify_attention(q, k, v)).float()
+    v[0, 0, -1, 5], v[0, 0, -1, 77] = float("inf"), float("-inf")
+    exp[..., 5], exp[..., 77] = float("inf"), float("-inf")
+    out = ops.gqa_decode(q.to(dev()), cache_buffer(k, kv_len + 9)[:, :, :kv_len],
+                         cache_buffer(v, kv_len + 9)[:, :, :kv_len]).cpu()
+    torch.testing.assert_close(out, exp, rtol=2e-5, atol=5e-5)
