@@ -101,6 +101,18 @@ def test_close_scores_fall_back_to_fp64():
         _check(q, k, P - T, torch.arange(P - T, dtype=torch.int32), k_sel)
 
 
+@pytest.mark.parametrize("T,P,k_sel", [(128, 9001, 3000), (20, 2500, 600)])
+def test_more_candidates_than_one_tile_a_workgroup(T, P, k_sel):
+    """Rows of 30 times the others' in one channel widen every bound: about a thousand
+    candidates, more than 16 for each workgroup of a head (split and fp64 statistics)."""
+    announce(f"bounded selection: many candidates T={T} P={P}")
+    gen = torch.Generator().manual_seed(T)
+    q = torch.randn(1, 28, T, 128, generator=gen)
+    q[:, ::7, :, 5] *= 30 if P > 5000 else 100
+    k = torch.randn(1, 4, P, 128, generator=gen)
+    _check(q.to(torch.bfloat16), k.to(torch.bfloat16), P - T, torch.arange(P - T, dtype=torch.int32), k_sel)
+
+
 def test_scattered_and_late_positions():
     """Gaps, positions inside the text rows (partly masked) and positions outside
     the prompt (score 0)."""
