@@ -286,26 +286,6 @@ __device__ __forceinline__ f32x4 load_part(const half_t* p) {
   return __builtin_convertvector(*reinterpret_cast<const half4_t*>(p), f32x4);
 }
 
-// Cross-lane max and sum of lanes l and l ^ 16 (xor16) or l and l ^ 32
-// (xor32) through v_permlane16/32_swap: both lanes get (the value of the one
-// with the bit clear) op (the value of the one with the bit set).
-__device__ __forceinline__ float xor16_max(float x) {
-  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-}
-__device__ __forceinline__ float xor32_max(float x) {
-  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-}
-__device__ __forceinline__ float xor16_sum(float x) {
-  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(a[0]) + __uint_as_float(a[1]);
-}
-__device__ __forceinline__ float xor32_sum(float x) {
-  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(a[0]) + __uint_as_float(a[1]);
-}
-
 // Merge, wave form (at most kWaveMergeMax splits: the draft's one-tile
 // splits, short verifies): one wave per row. Lane (c, h) = (lane & 31,
 // lane >> 5) owns columns 4c .. 4c + 3 and the splits h, h + 2, ..., h + 2(J-1)

@@ -50,6 +50,26 @@ template <> __device__ __forceinline__ f16_t from_f32<f16_t>(float x) { return (
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// Cross-lane max and sum of lanes l and l ^ 16 (xor16) or l and l ^ 32
+// (xor32) through v_permlane16/32_swap: both lanes get (the value of the one
+// with the bit clear) op (the value of the one with the bit set).
+__device__ __forceinline__ float xor16_max(float x) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+}
+__device__ __forceinline__ float xor32_max(float x) {
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+}
+__device__ __forceinline__ float xor16_sum(float x) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(a[0]) + __uint_as_float(a[1]);
+}
+__device__ __forceinline__ float xor32_sum(float x) {
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(a[0]) + __uint_as_float(a[1]);
+}
+
 // RMSNorm row statistic (modeling_qwen2_5_vl.py:192-197) in one fixed order,
 // shared by the norm kernel and the projection that normalises its own input:
 // over a block of 256 threads, thread t adds the squares of elements t,
