@@ -193,8 +193,10 @@ int std_verify_attn_append(const void* q, void* k_cache, void* v_cache,
  * token-major for the output projection). The caches already hold the n rows.
  * bf16 or fp16; any n >= 1, kv_len >= n, n_q a multiple of n_kv; scale > 0;
  * pointers 16-byte aligned and strides multiples of 8 elements. Scores,
- * probabilities and sums are fp32; each probability enters the PV product as a
- * 16-bit head plus a 16-bit remainder.
+ * probabilities and sums are fp32; a probability enters the PV product in 16-bit
+ * parts, in bf16 three that are the whole fp32 number, in fp16 two that leave at
+ * most one unit in its last place. A value that is not finite makes the outputs
+ * of the rows that see it, and of up to 63 rows before them, infinite or NaN.
  * ------------------------------------------------------------------------ */
 size_t std_prefill_attn_workspace_bytes(int n_q, int n_kv, int n, int kv_len, int d);
 
